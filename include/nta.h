@@ -468,7 +468,9 @@ int nta_pcg64_noalloc(const float* K, int n, long long ldk, double lam,
  *
  * nta_torus_tables: the normalisers of every layer for the n1 + n2 images
  * (from the images, or from slice (0, 0) of their self states): tables
- * [L][n1 + n2][nta_torus_table_floats(H, W, flags)].
+ * [L][n1 + n2][nta_torus_table_floats(H, W, flags)], with the powers of two by
+ * which an image's values are kept through the layers where its normalisers'
+ * squares would leave FP32's range.
  * nta_torus_pool: the segment followed by AvgPool 2x2 / 2, from the images
  * (in_nngp NULL) or a state, to the pooled state of size H/2 x W/2
  * (nta_torus_state_floats per pair).  band >= 0: only the pooled diagonals

@@ -192,7 +192,8 @@ __global__ __launch_bounds__(256) void k_flat_tables(
 // for equal rows) and h = sqrt(q1 q2), 1 - |rho| = s^2 / (h (h + |c|)) has no
 // cancellation, so theta = sqrt(1 - |rho|) P(|rho|) is accurate up to
 // |rho| = 1 with one reciprocal and two square roots (about 30 instructions
-// against 110 for atan2f and the IEEE square root).  a, b: (q, sqrt q).
+// against 110 for atan2f and the IEEE square root).  a, b: (q, sqrt q).  Its
+// hardware root and reciprocal take no subnormal s^2 or h^2: flat_plain.
 __device__ __forceinline__ float flat_relu(float c, float2 a, float2 b,
                                            float k1, float k0, float* ds) {
   const float d = fmaxf(prod_minus_sq(a.x, b.x, c), 0.0f);
@@ -206,11 +207,18 @@ __device__ __forceinline__ float flat_relu(float c, float2 a, float2 b,
   return fmaf(k1 * kInv2Pi, fmaf(pm, c, fsqrt(d)), k0 * c);
 }
 
+// Is a normaliser where flat_relu's products stay normal numbers (or 0, which
+// it treats apart)?  Otherwise a tile takes relu_map.
+__device__ __forceinline__ bool flat_plain(float q) {
+  return !(q > 0.0f && q < 0x1p-40f) && !(q > 0x1p40f);
+}
+
 // The network on E elements per thread.  qa(s, e), qb(s, e): normalisers
-// (q, sqrt q).
+// (q, sqrt q).  plain: flat_plain of all of them.
 template <int E, typename QA, typename QB>
-__device__ __forceinline__ void flat_chain(const FlatPlan& P, float (&n)[E],
-                                           float (&t)[E], QA qa, QB qb) {
+__device__ __forceinline__ void flat_chain(const FlatPlan& P, bool plain,
+                                           float (&n)[E], float (&t)[E],
+                                           QA qa, QB qb) {
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     n[e] *= P.inv_d;
@@ -225,7 +233,7 @@ __device__ __forceinline__ void flat_chain(const FlatPlan& P, float (&n)[E],
         t[e] = fmaf(S.w, t[e], n[e]);
       }
     }
-    if (S.act == NTA_RELU) {
+    if (S.act == NTA_RELU && plain) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         float ds;
@@ -277,12 +285,16 @@ __global__ __launch_bounds__(256) void k_flat_pairs(
   // The normalisers of the tile's rows and columns, in flight beside the
   // product: qs[stage][row | B + column].
   extern __shared__ float2 qs[];
+  __shared__ int odd;
+  if (threadIdx.x == 0) odd = 0;
+  __syncthreads();
   for (int k = threadIdx.x; k < P.nstage * 2 * B; k += 256) {
     const int s = k / (2 * B), o = k - s * (2 * B);
     if (P.s[s].act) {
       const float v =
           q[(long long)s * P.nimg + (o < B ? img_i(o) : img_j(o - B))];
       qs[k] = make_float2(v, fsqrt(fmaxf(v, 0.0f)));
+      if (!flat_plain(v)) odd = 1;
     }
   }
   // staged rows: the tile's rows, then its columns
@@ -297,7 +309,7 @@ __global__ __launch_bounds__(256) void k_flat_pairs(
 #pragma unroll
     for (int e = 0; e < 4; ++e) n[e] = tile[(r0 + 8 * e) * LP + c];
     flat_chain<4>(
-        P, n, t,
+        P, odd == 0, n, t,
         [&](int s, int e) { return qs[s * 2 * B + r0 + 8 * e]; },
         [&](int s, int) { return qs[s * 2 * B + B + c]; });
     __syncthreads();
@@ -320,7 +332,7 @@ __global__ __launch_bounds__(256) void k_flat_pairs(
       n[r] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
     auto row = [&](int r) { return wi + 8 * (r >> 2) + 4 * half + (r & 3); };
     flat_chain<16>(
-        P, n, t,
+        P, odd == 0, n, t,
         [&](int s, int r) { return qs[s * 2 * B + row(r)]; },
         [&](int s, int) { return qs[s * 2 * B + B + wj + col]; });
 #pragma unroll

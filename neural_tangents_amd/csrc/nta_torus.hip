@@ -127,6 +127,7 @@ int torus_fill(const char* who, TorusArgs& A, TorusGeom& g, int H, int W,
   A.RP = g.RP;
   A.PR = g.PR;
   A.TR = g.TR;
+  A.TS = g.TR * g.lw + 2;
   A.circ = circ;
   A.band = -1;
   *act = (flags & NTA_ACT_ERF) ? kActErf
@@ -286,7 +287,8 @@ extern "C" int nta_torus_supported(int H, int W, int C, int L, int pool,
 
 extern "C" long long nta_torus_table_floats(int H, int W, int flags) {
   TorusGeom g;
-  return torus_geom(H, W, 0, g, flags & NTA_TORUS_DIAG) ? 2LL * g.TR * g.lw : 0;
+  return torus_geom(H, W, 0, g, flags & NTA_TORUS_DIAG) ? 2LL * (g.TR * g.lw + 2)
+                                                        : 0;
 }
 
 extern "C" long long nta_torus_state_floats(int H, int W) {

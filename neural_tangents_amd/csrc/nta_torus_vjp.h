@@ -157,9 +157,18 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
       (jj ? xj : xi)[o] = torus_pixel(A, jj ? xb : xa, h, o - h * LW);
     }
   }
+  // The layers' constants for the pair's scaled values (nta_torus.h), their
+  // scales and those taken off again.
+  float we[L], be[L], ze[L], zr[L];
+#pragma unroll
   for (int l = 0; l < L; ++l) {
-    const float2* si = tab + ((long long)l * A.nimg + pr.i) * TR * LW;
-    const float2* sj = tab + ((long long)l * A.nimg + pr.j) * TR * LW;
+    const float2* si = tab + ((long long)l * A.nimg + pr.i) * A.TS;
+    const float2* sj = tab + ((long long)l * A.nimg + pr.j) * A.TS;
+    const TorusWB wb = torus_wb<true>(A, l, si[TR * LW], sj[TR * LW]);
+    we[l] = wb.w;
+    be[l] = wb.b;
+    ze[l] = wave_uniform(si[TR * LW].y * sj[TR * LW].y);
+    zr[l] = wave_uniform(torus_unscale<true>(si + TR * LW, sj + TR * LW));
     for (int q = tid; q < PR * LW; q += NT) ti[l * PR * LW + q] = si[q];
     for (int q = tid; q < TR * LW; q += NT) tj[l * TR * LW + q] = sj[q];
   }
@@ -192,10 +201,11 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
   const float* gpt = NTK && g_t ? g_t + (V.uniform ? pl : pl * per_out)
                                 : nullptr;
   const bool pooled = gpn && !V.uniform;
+  const float osc = V.osc * zr[L - 1];
   float un = 0.0f, ut = 0.0f;
   if (gpn && V.uniform) {
-    un = gpn[0] * V.osc;
-    if constexpr (NTK) ut = gpt[0] * V.osc;
+    un = gpn[0] * osc;
+    if constexpr (NTK) ut = gpt[0] * osc;
   }
 
   // The value at row r - 1 of an accumulator of image j (the row before this
@@ -249,10 +259,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
 #pragma unroll
       for (int l = 0; l < L; ++l) {
         const bool hu = NTK && (l > 0 || !IMG);
-        torus_stencil<LW, RS>(A, s, em, A.w[l], n);
-        if (hu) torus_stencil<LW, RS>(A, s, em, A.w[l], t);
+        torus_stencil<LW, RS>(A, s, em, we[l], n);
+        if (hu) torus_stencil<LW, RS>(A, s, em, we[l], t);
         if (l + 1 < L) {
-          const float bias = A.b[l], kk = A.k[l];
+          const float bias = be[l], kk = A.k[l];
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             park[(pk * R + r) * 64] = n[r];
@@ -288,7 +298,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
             v[q] = p[((q & 1) ? oo : oe) + ((r + q) >> 1) * go_h];
 #pragma unroll
           for (int q = 0; q < RB; ++q)
-            v[q] = ((q & 1) ? ok_o : ok_e) ? v[q] * V.osc : 0.0f;
+            v[q] = ((q & 1) ? ok_o : ok_e) ? v[q] * osc : 0.0f;
         } else {
 #pragma unroll
           for (int q = 0; q < RB; ++q) v[q] = head ? u : 0.0f;
@@ -300,10 +310,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
         const bool hu = NTK && (l > 0 || !IMG);
         if (l + 1 < L) {
           pk -= hu ? 2 : 1;
-          torus_stencil<LW, RS>(A, s, em, A.w[l + 1], n);
-          if constexpr (NTK) torus_stencil<LW, RS>(A, s, em, A.w[l + 1], t);
+          torus_stencil<LW, RS>(A, s, em, we[l + 1], n);
+          if constexpr (NTK) torus_stencil<LW, RS>(A, s, em, we[l + 1], t);
         }
-        const float bias = A.b[l], kk = A.k[l];
+        const float bias = be[l], kk = A.k[l];
         const float wrap = before(gb[l][R - 1]);
         float cn[RB], ct[RB];
 #pragma unroll
@@ -343,7 +353,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
             t[r] = gt;
           } else if (V.seeded) {
             if (s.vw)
-              gct += seed[((long long)pr.i * (L + (IMG ? A.C : 0)) + l) * S2 +
+              gct += zr[l] *
+                     seed[((long long)pr.i * (L + (IMG ? A.C : 0)) + l) * S2 +
                           (row0 + r) * H + w];
           }
           n[r] = gct;
@@ -358,8 +369,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
                          "+v"(sb[l]));
         }
       }
-      torus_stencil<LW, RS>(A, s, em, A.w[0], n);
-      if constexpr (!IMG && NTK) torus_stencil<LW, RS>(A, s, em, A.w[0], t);
+      torus_stencil<LW, RS>(A, s, em, we[0], n);
+      if constexpr (!IMG && NTK) torus_stencil<LW, RS>(A, s, em, we[0], t);
       if (live && s.vw) {
         const long long o =
             IMG ? ((pl * V.ne + job) * V.nd + dd) * S2 + row0 * H + w
@@ -403,14 +414,15 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_torus_vjp(
     if (live)
       for (int q = tid; q < Ks; q += NT) {
         const int l = q / S2, o = q - l * S2;
-        const float qv = tab[((long long)l * A.nimg + img) * TR * LW +
-                             o / H * LW + (o & (H - 1))].x;
-        out[side * Ks + q] = qv > 0.0f ? base[q] * 0.5f / qv : 0.0f;
+        const float2* tl = tab + ((long long)l * A.nimg + img) * A.TS;
+        const float qv = tl[o / H * LW + (o & (H - 1))].x;
+        const float z = tl[TR * LW].y;           // qv = z^2 q
+        out[side * Ks + q] = qv > 0.0f ? base[q] * 0.5f / qv * (z * z) : 0.0f;
       }
   }
 #pragma unroll
   for (int l = 0; l < L; ++l) {
-    double a = sw[l], b = sb[l];
+    double a = sw[l], b = sb[l] * (double)ze[l];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       a += __shfl_xor(a, o);
