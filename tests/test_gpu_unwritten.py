@@ -1,0 +1,92 @@
+"""Results do not depend on what stood in freshly allocated memory: every
+buffer that the package allocates is filled with NaN (needs a GPU).  Self
+chains leave the diagonals that no normaliser depends on unwritten."""
+import pytest
+import torch
+
+from neural_tangents_amd import grad, stax
+from neural_tangents_amd.data import blurred_images
+
+pytestmark = pytest.mark.gpu
+
+POOL = stax.AvgPool((2, 2), (2, 2))
+
+
+def _images(H, W, n=(3, 4)):
+  return [torch.from_numpy(x[:, :H, :W].copy()).cuda()
+          for x in blurred_images(list(n), max(H, W, 4), seed=H)]
+
+
+def _poison(monkeypatch):
+  empty, like = torch.empty, torch.empty_like
+
+  def fill(t):
+    return t.fill_(float('nan')) if t.is_floating_point() else t.fill_(255)
+  monkeypatch.setattr(torch, 'empty', lambda *a, **k: fill(empty(*a, **k)))
+  monkeypatch.setattr(torch, 'empty_like', lambda *a, **k: fill(like(*a,
+                                                                     **k)))
+
+
+def _same(got, want):
+  for g, w in zip(got, want):
+    assert torch.isfinite(w).all() and torch.equal(g, w)
+
+
+def _check(monkeypatch, kfn, H, W, get=('nngp', 'ntk')):
+  x1, x2 = _images(H, W)
+  for x in (x2, None):
+    want = kfn(x1, x, get)
+    with monkeypatch.context() as m:
+      _poison(m)
+      got = kfn(x1, x, get)
+    _same(got, want)
+    if get is None:
+      return
+    # and the values are those of an image alone with its partner
+    one = kfn(x1[2:], None if x is None else x[:1], get)
+    for g, o in zip(got, one):
+      torch.testing.assert_close(g[2:, 2 if x is None else 0].reshape(1, 1),
+                                 o, rtol=3e-7, atol=0.0)
+
+
+@pytest.mark.parametrize('side', list(range(8, 33)))
+@pytest.mark.parametrize('depths', [(2, 1, 1), (3, 3, 3)])
+def test_myrtle(monkeypatch, side, depths):
+  _check(monkeypatch, stax.myrtle(depths=list(depths))[2], side, side)
+
+
+@pytest.mark.parametrize('H,W', [(9, 13), (13, 8), (18, 11), (25, 32),
+                                 (32, 9)])
+@pytest.mark.parametrize('act', [stax.Relu(), stax.Erf(), stax.Gelu()])
+def test_pools_and_activations(monkeypatch, H, W, act):
+  c = [stax.Conv(1, (3, 3), padding='SAME', W_std=1.3, b_std=0.1), act]
+  kfn = stax.serial(*c, POOL, *c, POOL, *c, *c, stax.GlobalAvgPool(),
+                    stax.Dense(1))[2]
+  _check(monkeypatch, kfn, H, W)
+
+
+@pytest.mark.parametrize('side', [9, 16, 29])
+def test_readouts_without_pools(monkeypatch, side):
+  c = [stax.Conv(1, (3, 3), padding='SAME', W_std=1.3), stax.Relu()] * 3
+  for head in (stax.GlobalAvgPool(), stax.Flatten()):
+    _check(monkeypatch, stax.serial(*c, head, stax.Dense(1))[2], side, side)
+
+
+@pytest.mark.parametrize('side', [8, 16, 32])
+@pytest.mark.parametrize('same', [True, False])
+def test_gradients(monkeypatch, side, same):
+  xs = _images(side, side)
+
+  def run():
+    a, b = (x.clone().requires_grad_() for x in xs)
+    W = torch.tensor(1.4, device='cuda', requires_grad=True)
+    k = grad.kernel(a, None if same else b, W, 0.1,
+                    grad.myrtle_builder((2, 1, 1)))
+    gs = torch.autograd.grad((k[0] + k[1]).sum(),
+                             (a, W) if same else (a, b, W))
+    return k + gs
+  want = run()
+  with monkeypatch.context() as m:
+    _poison(m)
+    got = run()
+  _same(got, want)
