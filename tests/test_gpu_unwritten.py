@@ -65,6 +65,15 @@ def test_pools_and_activations(monkeypatch, H, W, act):
   _check(monkeypatch, kfn, H, W)
 
 
+@pytest.mark.parametrize('side', [8, 16, 24, 32])
+def test_periodic(monkeypatch, side):
+  c = [stax.Conv(1, (3, 3), padding='CIRCULAR', W_std=1.3, b_std=0.1),
+       stax.Relu()]
+  kfn = stax.serial(*c, *c, POOL, *c, POOL, *c, stax.GlobalAvgPool(),
+                    stax.Dense(1))[2]
+  _check(monkeypatch, kfn, side, side)
+
+
 @pytest.mark.parametrize('side', [9, 16, 29])
 def test_readouts_without_pools(monkeypatch, side):
   c = [stax.Conv(1, (3, 3), padding='SAME', W_std=1.3), stax.Relu()] * 3
