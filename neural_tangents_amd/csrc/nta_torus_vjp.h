@@ -45,7 +45,7 @@ __device__ __forceinline__ VjpAngle vjp_angle(float c, float2 qa, float2 qb,
   const float d = prod_minus_sq(qa.x, qb.x, c) * keep;
   r.rs = d > 1.2e-38f ? __builtin_amdgcn_rsqf(d) : 0.0f;
   r.s = d * r.rs;
-  float h = fmaf(-(r.s * rh), acos_over_sin<8>(a), 0.5f * kPi);
+  float h = fmaf(-(r.s * rh), acos_over_sin<9>(a), 0.5f * kPi);
   h = rh > 0.0f ? h : 0.0f;             // no variance: theta = pi / 2
   r.pk = (0.5f * kPi + copysignf(h, rho)) + k;
   return r;
