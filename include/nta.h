@@ -49,7 +49,7 @@ extern "C" {
 #define NTA_ACT_GELU 64   /* Gelu (act_k1, act_k0 unused)                   */
 #define NTA_TORUS_SELF 256   /* nta_torus_*: pairs are images with themselves */
 #define NTA_TORUS_DIAG 1024  /* nta_torus_*: the table layout of nta_torus_diag */
-#define NTA_TORUS_EXACT 2048 /* nta_torus_tables: (q, 1 / sqrt q) always */
+#define NTA_TORUS_EXACT 2048 /* nta_torus_tables: not for nta_torus_pool   */
 #define NTA_TORUS_UPPER 512  /* nta_torus_*, nta_flat_*: x1 with x1, upper half */
 
 /* Library version (major*10000 + minor*100 + patch). */
@@ -468,9 +468,10 @@ int nta_pcg64_noalloc(const float* K, int n, long long ldk, double lam,
  *
  * nta_torus_tables: the normalisers of every layer for the n1 + n2 images
  * (from the images, or from slice (0, 0) of their self states): tables
- * [L][n1 + n2][nta_torus_table_floats(H, W, flags)], with the powers of two by
- * which an image's values are kept through the layers where its normalisers'
- * squares would leave FP32's range.
+ * [L][n1 + n2][nta_torus_table_floats(H, W, flags)], made with NTA_TORUS_EXACT
+ * in flags for nta_torus_gap and nta_torus_vjp, without for nta_torus_pool.
+ * They hold the powers of two by which an image's values are kept through the
+ * layers where its normalisers' squares would leave FP32's range.
  * nta_torus_pool: the segment followed by AvgPool 2x2 / 2, from the images
  * (in_nngp NULL) or a state, to the pooled state of size H/2 x W/2
  * (nta_torus_state_floats per pair).  band >= 0: only the pooled diagonals

@@ -982,7 +982,8 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
   for k, s in enumerate(segs):
     tab = empty(s.L, nimg, _lib.value('nta_torus_table_floats', s.H, s.W, 0))
     _launch('nta_torus_tables', 4 * tab.numel(), 0, px1, px2, N1, N2,
-            _lib.ptr(st), s.H, s.W, C, s.L, s.wb, s.flags, _lib.ptr(tab),
+            _lib.ptr(st), s.H, s.W, C, s.L, s.wb,
+            s.flags | (0 if s.pool else _lib.TORUS_EXACT), _lib.ptr(tab),
             0.0, 0.0, None, stream)
     tabs.append(tab)
     if s.pool:

@@ -162,9 +162,8 @@ int torus_fill(const char* who, TorusArgs& A, TorusGeom& g, int H, int W,
     }
   }
   A.out_scale = scale;
-  // as torus_map: the sizes with a correlation-form instance
-  const bool pow2 = H == W && (H == 16 || H == 32);
-  A.exact = !(*act == kActRelu && !circ && pow2 &&
+  // as torus_map: the size with a correlation-form instance
+  A.exact = !(*act == kActRelu && !circ && H == 32 && W == 32 &&
               !(flags & (NTA_TORUS_DIAG | NTA_TORUS_EXACT)));
   return NTA_OK;
 }
@@ -418,7 +417,8 @@ extern "C" int nta_torus_gap(const float* x1, const float* x2, int n1, int n2,
   int act;
   const bool img = in_nngp == nullptr;
   const bool ntk = (flags & NTA_NTK) && !(flags & NTA_TORUS_SELF);
-  int rc = torus_fill("nta_torus_gap", A, g, H, W, C, img, L, wb, flags, &act);
+  int rc = torus_fill("nta_torus_gap", A, g, H, W, C, img, L, wb,
+                      flags | NTA_TORUS_EXACT, &act);
   if (rc) return rc;
   rc = torus_set_pairs("nta_torus_gap", A, n1, n2, flags, p0, np);
   if (rc) return rc;
