@@ -359,7 +359,7 @@ extern "C" int nta_torus_pool(const float* x1, const float* x2, int n1,
     return set_error(NTA_EINVAL, "nta_torus_pool: %dx%d does not pool", H, W);
   if (np == 0) return NTA_OK;
   if (!tables || !out_nngp || (ntk && !out_ntk) ||
-      (img ? (!x1 || (n2 > 0 && !x2)) : (ntk && !in_ntk)))
+      (img ? ((n1 > 0 && !x1) || (n2 > 0 && !x2)) : (ntk && !in_ntk)))
     return set_error(NTA_EINVAL, "nta_torus_pool: null pointer");
   A.Ho = H / 2;
   A.Wo = W / 2;
@@ -430,7 +430,7 @@ extern "C" int nta_torus_gap(const float* x1, const float* x2, int n1, int n2,
   A.Wc = crop_w;
   choose_chunks(A, g);
   if (!tables || !out_nngp || (ntk && !out_ntk) || !work ||
-      (img ? (!x1 || (n2 > 0 && !x2)) : (ntk && !in_ntk)))
+      (img ? ((n1 > 0 && !x1) || (n2 > 0 && !x2)) : (ntk && !in_ntk)))
     return set_error(NTA_EINVAL, "nta_torus_gap: null pointer");
   if (work_bytes < 16 * np * A.nchunk)
     return set_error(NTA_EINVAL, "nta_torus_gap: work of %lld bytes",

@@ -173,7 +173,7 @@ extern "C" int nta_torus_vjp(const float* x1, const float* x2, int n1, int n2,
   if (np == 0) return NTA_OK;
   if (!tables || !acc || !wb_acc || !work || (!self && !g_nngp) ||
       (ntk && !g_ntk) ||
-      (img ? (!x1 || (n2 > 0 && !x2))
+      (img ? ((n1 > 0 && !x1) || (n2 > 0 && !x2))
            : (!gin_nngp || (ntk && (!in_ntk || !gin_ntk)))))
     return set_error(NTA_EINVAL, "nta_torus_vjp: null pointer");
   VjpArgs V = VjpArgs();
