@@ -949,12 +949,91 @@ def _torus_segments(plan: Plan, in_shape) -> Optional[List[Segment]]:
   return segs or None
 
 
+def _torus_bands(segs) -> List[int]:
+  """Diagonals |d| <= band of the self states after each pooled segment that
+  later normalisers depend on: the last segment's need the diagonal, a pooled
+  diagonal d the input's 2d - 1, 2d, 2d + 1."""
+  band = [0] * len(segs)
+  for k in range(len(segs) - 3, -1, -1):
+    band[k] = 2 * band[k + 1] + 1
+  return band
+
+
+def _torus_state(n, seg, dev):
+  """An empty state of n pairs before seg."""
+  return torch.empty((n, _lib.value('nta_torus_state_floats', seg.H, seg.W)),
+                     dtype=torch.float32, device=dev)
+
+
+def _torus_tables(segs, n, dev):
+  """Empty normaliser tables of n images, per segment."""
+  return [torch.empty((s.L, n, _lib.value('nta_torus_table_floats', s.H, s.W,
+                                          0)),
+                      dtype=torch.float32, device=dev) for s in segs]
+
+
+def _torus_images(x1, x2, most):
+  """(x1 part, x2 part, index of the first image, images) with at most
+  ``most`` images each: all of them, or runs of one argument."""
+  N1 = x1.shape[0]
+  N2 = 0 if x2 is None else x2.shape[0]
+  if N1 + N2 <= most:
+    return [(x1, x2, 0, N1 + N2)]
+  return [(x[i:i + most], None, at + i, min(most, x.shape[0] - i))
+          for x, at in ((x1, 0), (x2, N1)) if x is not None
+          for i in range(0, x.shape[0], most)]
+
+
+def _torus_selfs(segs, x1, x2, stream, coef=None, adjoint=False):
+  """Self chains of the images of x1 and x2.  Returns the normaliser tables
+  per segment, those of the adjoint (None without ``adjoint``), the states
+  before the segments (None for the first) and the self covariances of the
+  readout ``coef`` (None without).  Of the states only the diagonals that
+  later normalisers depend on are computed, unless the readout is asked
+  for."""
+  dev = x1.device
+  N1, _, _, C = x1.shape
+  N2 = 0 if x2 is None else x2.shape[0]
+  n = N1 + N2
+  px = (_lib.ptr(x1), _lib.ptr(x2), N1, N2)
+  band = _torus_bands(segs)
+  tabs = _torus_tables(segs, n, dev)
+  xtabs = _torus_tables(segs, n, dev) if adjoint else None
+  states, cov = [None], None
+  for k, s in enumerate(segs):
+    st = _lib.ptr(states[k])
+
+    def tables(dst, flag):
+      _launch('nta_torus_tables', 4 * dst.numel(), 0, *px, st, s.H, s.W, C,
+              s.L, s.wb, s.flags | flag, _lib.ptr(dst), 0.0, 0.0, None,
+              stream)
+    tables(tabs[k], 0 if s.pool else _lib.TORUS_EXACT)
+    if adjoint:
+      tables(xtabs[k], _lib.TORUS_EXACT)
+    if s.pool:
+      states.append(_torus_state(n, segs[k + 1], dev))
+      _launch(f'nta_torus_pool[self {s.H}]', n * s.layer_bytes(k == 0), n,
+              *px, 0, n, st, None, s.H, s.W, C, s.L, s.wb,
+              s.flags | _lib.TORUS_SELF, -1 if coef else band[k],
+              _lib.ptr(tabs[k]), _lib.ptr(states[k + 1]), None, stream)
+      if not adjoint:
+        states[k] = None
+    elif coef:
+      cov = torch.empty((n,), dtype=torch.float32, device=dev)
+      nw = _lib.value('nta_torus_gap_work_bytes', s.H, s.W, n)
+      work = torch.empty((nw,), dtype=torch.uint8, device=dev)
+      _launch(f'nta_torus_gap[self {s.H}]', n * s.layer_bytes(k == 0), n,
+              *px, 0, n, st, None, s.H, s.W, C, s.L, s.wb,
+              s.flags | _lib.TORUS_SELF, *s.crop, _lib.ptr(tabs[k]), *coef,
+              _lib.ptr(cov), None, 0, _lib.ptr(work), nw, stream)
+  return tabs, xtabs, states, cov
+
+
 def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
                stream, keep=None):
-  """Runs the segments: the self chains of all images (x1, then x2) leave
+  """Runs the segments: the self chains of the images (x1, then x2) leave
   every layer's normaliser tables, then the pairs (the upper triangle when
-  x2 is None) in tiles.  Of the self states only the diagonals that later
-  normalisers depend on are computed, unless their readout is asked for.
+  x2 is None); both in tiles whose states take at most tile_bytes.
   keep: a list that receives the (nngp, ntk) states of all pairs before every
   segment but the first, if they are one tile of at most KEEP_BYTES."""
   dev = x1.device
@@ -968,41 +1047,26 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
     return torch.empty(shape, dtype=torch.float32, device=dev)
 
   def state(n, seg):
-    return empty(n, _lib.value('nta_torus_state_floats', seg.H, seg.W))
+    return _torus_state(n, seg, dev)
 
-  # bands of the self states after each pooled segment: the last segment's
-  # normalisers need the diagonal, a pooled diagonal d the input's 2d - 1,
-  # 2d, 2d + 1
-  band = [0] * len(segs)
-  for k in range(len(segs) - 3, -1, -1):
-    band[k] = 2 * band[k + 1] + 1
-  tabs = []
-  st = None
-  cov = None
-  for k, s in enumerate(segs):
-    tab = empty(s.L, nimg, _lib.value('nta_torus_table_floats', s.H, s.W, 0))
-    _launch('nta_torus_tables', 4 * tab.numel(), 0, px1, px2, N1, N2,
-            _lib.ptr(st), s.H, s.W, C, s.L, s.wb,
-            s.flags | (0 if s.pool else _lib.TORUS_EXACT), _lib.ptr(tab),
-            0.0, 0.0, None, stream)
-    tabs.append(tab)
-    if s.pool:
-      out = state(nimg, segs[k + 1])
-      _launch(f'nta_torus_pool[self {s.H}]', nimg * s.layer_bytes(k == 0),
-              nimg, px1, px2, N1, N2, 0, nimg, _lib.ptr(st), None, s.H, s.W,
-              C, s.L, s.wb, s.flags | _lib.TORUS_SELF,
-              -1 if want_cov else band[k], _lib.ptr(tab), _lib.ptr(out),
-              None, stream)
-      st = out
-    elif want_cov:
-      cov = empty(nimg)
-      nw = _lib.value('nta_torus_gap_work_bytes', s.H, s.W, nimg)
-      work = torch.empty((nw,), dtype=torch.uint8, device=dev)
-      _launch(f'nta_torus_gap[self {s.H}]', nimg * s.layer_bytes(k == 0),
-              nimg, px1, px2, N1, N2, 0, nimg, _lib.ptr(st), None, s.H, s.W,
-              C, s.L, s.wb, s.flags | _lib.TORUS_SELF, *s.crop,
-              _lib.ptr(tab), a, b, c, d, e, _lib.ptr(cov), None, 0,
-              _lib.ptr(work), nw, stream)
+  # a segment's input and output state
+  floats = [0] + [_lib.value('nta_torus_state_floats', s.H, s.W)
+                  for s in segs[1:]] + [0]
+  most = max(1, tile_bytes // max(1, 4 * max(map(sum, zip(floats,
+                                                          floats[1:])))))
+  coef = plan.head_coef if want_cov else None
+  parts = _torus_images(x1, x2, most)
+  if len(parts) == 1:
+    tabs, _, _, cov = _torus_selfs(segs, x1, x2, stream, coef)
+  else:
+    tabs = _torus_tables(segs, nimg, dev)
+    cov = empty(nimg) if want_cov else None
+    for xa, xb, at, n in parts:
+      part, _, _, pcov = _torus_selfs(segs, xa, xb, stream, coef)
+      for t, p in zip(tabs, part):
+        t[:, at:at + n] = p
+      if want_cov:
+        cov[at:at + n] = pcov
   cols = N1 if x2 is None else N2
   nngp = empty(N1, cols)
   ntk = empty(N1, cols) if want_ntk else None

@@ -1,0 +1,46 @@
+"""Self chains of many images keep to their memory, and give what they give
+all at once (needs a GPU)."""
+import pytest
+import torch
+
+from neural_tangents_amd import stax
+from neural_tangents_amd.data import blurred_images
+
+pytestmark = pytest.mark.gpu
+
+
+def _images(n, side, seed):
+  return torch.from_numpy(blurred_images([n], side, seed=seed)[0]).cuda()
+
+
+@pytest.mark.parametrize('side', [9, 16, 32])
+@pytest.mark.parametrize('get', [('nngp', 'ntk'), None])
+@pytest.mark.parametrize('same', [True, False])
+def test_tiles_of_images(side, get, same):
+  """One ulp of the mean: the pairs of a tile may be split in other shares."""
+  kfn = stax.myrtle(5)[2]
+  x1, x2 = _images(5, side, 1), None if same else _images(4, side, 2)
+  want = kfn(x1, x2, get)
+  per = 4 * 2 * (side // 2 + 1) ** 4
+  got = kfn(x1, x2, get, tile_bytes=2 * per)
+  fields = get or ('nngp', 'ntk', 'cov1') + (() if same else ('cov2',))
+  for f in fields:
+    torch.testing.assert_close(getattr(got, f), getattr(want, f),
+                               rtol=1.2e-7, atol=0.0)
+
+
+@pytest.mark.parametrize('get', [('nngp', 'ntk'), None])
+def test_tile_bytes_bounds_the_states(get):
+  """400 images of 32x32 have 100 MiB of pooled self states; within 4 MiB of
+  tiles only the tables (32 KiB + 4 KiB + 1 KiB an image, once for the part
+  at hand) and the results are more."""
+  kfn = stax.myrtle(5)[2]
+  x1, x2 = _images(400, 32, 1), _images(1, 32, 2)
+  kfn(x1[:2], x2, get, tile_bytes=1 << 22)
+  torch.cuda.synchronize()
+  torch.cuda.empty_cache()
+  before = torch.cuda.memory_allocated()
+  torch.cuda.reset_peak_memory_stats()
+  kfn(x1, x2, get, tile_bytes=1 << 22)
+  peak = torch.cuda.max_memory_allocated() - before
+  assert peak <= (2 << 22) + 401 * (40 << 10) + (8 << 20), peak
