@@ -260,6 +260,11 @@ def kernel_vjp(plan, x1, x2, g_nngp, g_ntk, tile_pairs=512, states=()):
           [float(v) for v in sums[L:]])
 
 
+# States and workspaces of the self chains' adjoints that are held at a time
+# (0.8 MiB a 32x32 image).
+SELF_BYTES = 2 << 30
+
+
 def _torus_segments(plan, in_shape):
   """The segments of a network that nta_torus_vjp covers, else None."""
   segs = _engine._torus_segments(plan, in_shape)
@@ -289,20 +294,18 @@ def _torus_vjp(plan, segs, x1, x2, g_nngp, g_ntk, tile_pairs, kept):
   px = (_lib.ptr(x1), _lib.ptr(x2), N1, N2)
   K = len(segs)
 
-  def empty(*shape):
-    return torch.empty(shape, dtype=torch.float32, device=dev)
-
-  def state(n, s):
-    return empty(n, _lib.value('nta_torus_state_floats', s.H, s.W))
-
-  def adjoint(k, p0, T, states, flags, band, g, uniform, gin):
+  def work_bytes(k, T, band):
     s = segs[k]
-    c = 0 if k else C
-    nw = _lib.value('nta_torus_vjp_work_bytes', s.H, c, s.L, T, band)
+    return _lib.value('nta_torus_vjp_work_bytes', s.H, 0 if k else C, s.L, T,
+                      band)
+
+  def adjoint(k, px, p0, T, states, flags, band, tab, g, uniform, gin, acc):
+    s = segs[k]
+    nw = work_bytes(k, T, band)
     work = torch.empty((nw,), dtype=torch.uint8, device=dev)
-    _lib.call('nta_torus_vjp', *px, p0, T, *map(_lib.ptr, states), s.H, c,
-              s.L, s.wb, flags, band, _lib.ptr(tabs[k]), *map(_lib.ptr, g),
-              uniform, *map(_lib.ptr, gin), _lib.ptr(acc[k]),
+    _lib.call('nta_torus_vjp', *px, p0, T, *map(_lib.ptr, states), s.H,
+              0 if k else C, s.L, s.wb, flags, band, _lib.ptr(tab),
+              *map(_lib.ptr, g), uniform, *map(_lib.ptr, gin), _lib.ptr(acc),
               _lib.ptr(wb[first[k]]), _lib.ptr(work), nw, stream)
 
   def none_or(cotangent):
@@ -318,26 +321,28 @@ def _torus_vjp(plan, segs, x1, x2, g_nngp, g_ntk, tile_pairs, kept):
   gm = (g_n.mul(a / nlast).add_(g_t, alpha=c / nlast).reshape(-1),
         g_t.mul(d / nlast).reshape(-1).contiguous())
   # self chains: the kernels' normaliser tables, the adjoint's (q itself) and
-  # the self states on the diagonals that later normalisers depend on
-  band = [0] * K
-  for k in range(K - 3, -1, -1):
-    band[k] = 2 * band[k + 1] + 1
+  # the self states on the diagonals that later normalisers depend on, of as
+  # many images at a time as their states and adjoints take SELF_BYTES
+  band = [b if s.pool else -1
+          for b, s in zip(_engine._torus_bands(segs), segs)]
   first = [sum(s.L for s in segs[:k]) for k in range(K)]
-  ftabs, tabs, selfs, acc = [], [], [None], []
-  for k, s in enumerate(segs):
-    shape = (s.L, nimg, _lib.value('nta_torus_table_floats', s.H, s.W, 0))
-    for dst, flag in ((ftabs, 0), (tabs, _lib.TORUS_EXACT)):
-      dst.append(empty(*shape))
-      _lib.call('nta_torus_tables', *px, _lib.ptr(selfs[k]), s.H, s.W, C,
-                s.L, s.wb, s.flags | flag, _lib.ptr(dst[k]), 0.0, 0.0, None,
-                stream)
-    acc.append(torch.zeros((nimg, s.L + (0 if k else C), s.H * s.W),
-                           dtype=torch.float32, device=dev))
-    if s.pool:
-      selfs.append(state(nimg, segs[k + 1]))
-      _lib.call('nta_torus_pool', *px, 0, nimg, _lib.ptr(selfs[k]), None,
-                s.H, s.W, C, s.L, s.wb, s.flags | _lib.TORUS_SELF, band[k],
-                _lib.ptr(ftabs[k]), _lib.ptr(selfs[k + 1]), None, stream)
+  per = sum(work_bytes(k, 1, band[k]) + 8 * _lib.value(
+      'nta_torus_state_floats', s.H, s.W) * (k > 0)
+      for k, s in enumerate(segs))
+  parts = _engine._torus_images(x1, x2, max(1, SELF_BYTES // per))
+  if len(parts) == 1:
+    ftabs, tabs, selfs, _ = _engine._torus_selfs(segs, x1, x2, stream,
+                                                 adjoint=True)
+  else:
+    ftabs, tabs = (_engine._torus_tables(segs, nimg, dev) for _ in range(2))
+    for xa, xb, at, n in parts:
+      part = _engine._torus_selfs(segs, xa, xb, stream, adjoint=True)
+      for dst, src in zip(ftabs + tabs, part[0] + part[1]):
+        dst[:, at:at + n] = src
+    del part
+  acc = [torch.zeros((nimg, s.L + (0 if k else C), s.H * s.W),
+                     dtype=torch.float32, device=dev)
+         for k, s in enumerate(segs)]
   wb = torch.zeros((len(plan.stages), 2), dtype=torch.float64, device=dev)
   mode = _lib.NTK | (_lib.TORUS_UPPER if sym else 0)
   pairs = N1 * (N1 + 1) // 2 if sym else N1 * N2
@@ -347,7 +352,8 @@ def _torus_vjp(plan, segs, x1, x2, g_nngp, g_ntk, tile_pairs, kept):
     states = [(None, None)] + [tuple(t[p0:p0 + T] for t in pair)
                                for pair in kept]
     for k, s in enumerate(() if kept else segs[:-1]):
-      states.append((state(T, segs[k + 1]), state(T, segs[k + 1])))
+      states.append(tuple(_engine._torus_state(T, segs[k + 1], dev)
+                          for _ in range(2)))
       _lib.call('nta_torus_pool', *px, p0, T, *map(_lib.ptr, states[k]), s.H,
                 s.W, C, s.L, s.wb, s.flags | mode, -1, _lib.ptr(ftabs[k]),
                 *map(_lib.ptr, states[k + 1]), stream)
@@ -355,15 +361,22 @@ def _torus_vjp(plan, segs, x1, x2, g_nngp, g_ntk, tile_pairs, kept):
     for k in range(K - 1, -1, -1):
       gin = (None, None) if k == 0 else tuple(map(torch.empty_like,
                                                   states[k]))
-      adjoint(k, p0, T, states[k], segs[k].flags | mode, -1, g,
-              int(k == K - 1), gin)
+      adjoint(k, px, p0, T, states[k], segs[k].flags | mode, -1, tabs[k], g,
+              int(k == K - 1), gin, acc[k])
       g = gin
-  g = (None, None)
-  for k in range(K - 1, -1, -1):
-    gin = (None if k == 0 else torch.empty_like(selfs[k]), None)
-    adjoint(k, 0, nimg, (selfs[k], None), segs[k].flags | _lib.TORUS_SELF,
-            band[k] if segs[k].pool else -1, g, 0, gin)
-    g = gin
+  for xa, xb, at, n in parts:
+    if len(parts) > 1:
+      _, tabs, selfs, _ = _engine._torus_selfs(segs, xa, xb, stream,
+                                               adjoint=True)
+    pa = (_lib.ptr(xa), _lib.ptr(xb), xa.shape[0],
+          0 if xb is None else xb.shape[0])
+    g = (None, None)
+    for k in range(K - 1, -1, -1):
+      gin = (None if k == 0 else torch.empty_like(selfs[k]), None)
+      adjoint(k, pa, 0, n, (selfs[k], None),
+              segs[k].flags | _lib.TORUS_SELF, band[k], tabs[k], g, 0, gin,
+              acc[k][at:at + n])
+      g = gin
   gx = acc[0][:, segs[0].L:].reshape((nimg,) + tuple(x1.shape[1:]))
   sums = wb.cpu()                                            # one sync
   return (gx[:N1].contiguous(), None if sym else gx[N1:].contiguous(),

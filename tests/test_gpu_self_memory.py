@@ -3,7 +3,7 @@ all at once (needs a GPU)."""
 import pytest
 import torch
 
-from neural_tangents_amd import stax
+from neural_tangents_amd import grad, stax
 from neural_tangents_amd.data import blurred_images
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +44,37 @@ def test_tile_bytes_bounds_the_states(get):
   kfn(x1, x2, get, tile_bytes=1 << 22)
   peak = torch.cuda.max_memory_allocated() - before
   assert peak <= (2 << 22) + 401 * (40 << 10) + (8 << 20), peak
+
+
+@pytest.mark.parametrize('side', [8, 32])
+@pytest.mark.parametrize('same', [True, False])
+def test_gradients_in_parts(monkeypatch, side, same):
+  """Images' cotangents do not mix, so theirs are the same bit for bit; the
+  FP64 sums for W_std and b_std come in another order."""
+  xs = [_images(5, side, 1), _images(4, side, 2)]
+
+  def run():
+    a, b = (x.clone().requires_grad_() for x in xs)
+    W, bs = (torch.tensor(v, device='cuda', requires_grad=True)
+             for v in (1.4, 0.1))
+    n, t = grad.kernel(a, None if same else b, W, bs,
+                       grad.myrtle_builder((2, 1, 1)))
+    return torch.autograd.grad((n + t).sum(), [a, W, bs] +
+                               ([] if same else [b]))
+  want = run()
+  with monkeypatch.context() as m:
+    parts = []
+    images = grad._engine._torus_images
+
+    def record(*a):
+      parts.append(images(*a))
+      return parts[-1]
+    m.setattr(grad._engine, '_torus_images', record)
+    m.setattr(grad, 'SELF_BYTES', 1)
+    got = run()
+  assert any(len(p) == (5 if same else 9) for p in parts)
+  for k, (g, w) in enumerate(zip(got, want)):
+    if k in (1, 2):
+      assert abs(float(g) - float(w)) <= 1e-12 * abs(float(w))
+    else:
+      assert torch.equal(g, w)
