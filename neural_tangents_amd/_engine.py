@@ -24,9 +24,11 @@ Reference call path replaced: ``_preprocess_kernel_fn`` /
 import dataclasses
 import functools
 import math
+import threading
 from typing import List, Optional, Tuple
 
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from . import _lib
 
@@ -334,9 +336,36 @@ def compile_plan(specs, in_shape, from_state: bool = False,
 # ------------------------------------------------------------------ runner
 
 DEFAULT_TILE_BYTES = 6 << 30
-# Pair states that a differentiated call leaves for its backward (0.5 MiB a
-# 32x32 pair), which otherwise computes them again.
+# Pair states that differentiated calls leave for their backward (0.5 MiB a
+# 32x32 pair), which otherwise computes them again: at most this much on a
+# device, of all calls whose graphs are alive.
 KEEP_BYTES = 4 << 30
+_kept_lock = threading.Lock()
+_kept = {}                # device -> [bytes, [(weak storage, bytes)]]
+
+
+def _kept_states(segs, pairs, want_ntk, dev):
+  """Empty (nngp, ntk) states of all pairs before every segment but the first,
+  counted against KEEP_BYTES while anything holds them, or None if there is no
+  room."""
+  sizes = [_lib.value('nta_torus_state_floats', s.H, s.W) for s in segs[1:]]
+  need = 4 * pairs * sum(sizes) * (2 if want_ntk else 1)
+  with _kept_lock:
+    entry = _kept.setdefault(dev, [0, []])
+    if entry[0] + need > KEEP_BYTES:
+      entry[1] = [e for e in entry[1] if not e[0].expired()]
+      entry[0] = sum(n for _, n in entry[1])
+      if entry[0] + need > KEEP_BYTES:
+        return None
+    out = []
+    for s in segs[1:]:
+      pair = [_torus_state(pairs, s, dev) for _ in range(1 + want_ntk)]
+      for t in pair:
+        n = 4 * t.numel()
+        entry[0] += n
+        entry[1].append((StorageWeakRef(t.untyped_storage()), n))
+      out.append((pair[0], pair[1] if want_ntk else None))
+  return out
 
 # When a list, every launch appends (entry point, start event, end event,
 # algorithmic HBM bytes of the launch, pairs in the launch).  Used by the
@@ -1035,7 +1064,8 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
   every layer's normaliser tables, then the pairs (the upper triangle when
   x2 is None); both in tiles whose states take at most tile_bytes.
   keep: a list that receives the (nngp, ntk) states of all pairs before every
-  segment but the first, if they are one tile of at most KEEP_BYTES."""
+  segment but the first, if they are one tile and there is room
+  (_kept_states)."""
   dev = x1.device
   N1, H, W, C = x1.shape
   N2 = 0 if x2 is None else x2.shape[0]
@@ -1077,30 +1107,31 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
   per = max([4 * nt * 2 * _lib.value('nta_torus_state_floats', s.H, s.W)
              for s in segs[1:]], default=0)
   tile = min(pairs, max(1, tile_bytes // per) if per else 1 << 20)
-  if keep is not None and (tile < pairs or pairs * sum(
-      4 * nt * _lib.value('nta_torus_state_floats', s.H, s.W)
-      for s in segs[1:]) > KEEP_BYTES):
-    keep = None
+  held = None
+  if keep is not None and tile == pairs:
+    held = _kept_states(segs, pairs, want_ntk, dev)
+    keep.extend(held or ())
   for p0 in range(0, pairs, max(tile, 1)):
     T = min(tile, pairs - p0)
     sn = stt = None
     for k, s in enumerate(segs):
       if s.pool:
-        on = state(T, segs[k + 1])
-        ot = torch.empty_like(on) if want_ntk else None
+        if held is not None:
+          on, ot = held[k]
+        else:
+          on = state(T, segs[k + 1])
+          ot = torch.empty_like(on) if want_ntk else None
         _launch(f'nta_torus_pool[{s.H}]', T * nt * s.layer_bytes(k == 0), T,
-                px1, px2, N1, N2, p0, T, _lib.ptr(sn), _lib.ptr(stt), s.H, s.W, C, s.L, s.wb,
-                s.flags | mode, -1, _lib.ptr(tabs[k]), _lib.ptr(on),
-                _lib.ptr(ot), stream)
+                px1, px2, N1, N2, p0, T, _lib.ptr(sn), _lib.ptr(stt), s.H,
+                s.W, C, s.L, s.wb, s.flags | mode, -1, _lib.ptr(tabs[k]),
+                _lib.ptr(on), _lib.ptr(ot), stream)
         sn, stt = on, ot
-        if keep is not None:
-          keep.append((on, ot))
       else:
         nw = _lib.value('nta_torus_gap_work_bytes', s.H, s.W, T)
         work = torch.empty((nw,), dtype=torch.uint8, device=dev)
         _launch(f'nta_torus_gap[{s.H}]', T * nt * s.layer_bytes(k == 0), T,
-                px1, px2, N1, N2, p0, T, _lib.ptr(sn), _lib.ptr(stt), s.H, s.W, C, s.L, s.wb,
-                s.flags | mode, *s.crop, _lib.ptr(tabs[k]), a, b, c, d, e,
+                px1, px2, N1, N2, p0, T, _lib.ptr(sn), _lib.ptr(stt), s.H,
+                s.W, C, s.L, s.wb, s.flags | mode, *s.crop, _lib.ptr(tabs[k]), a, b, c, d, e,
                 _lib.ptr(nngp), _lib.ptr(ntk), cols, _lib.ptr(work), nw,
                 stream)
   return {'cov1': None if cov is None else cov[:N1],

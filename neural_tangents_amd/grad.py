@@ -448,14 +448,16 @@ def _self_chain_vjp(plan, x, gq, gx, gwv, gbv, stream, C, fh, fw,
 class KernelFunction(torch.autograd.Function):
   """(nngp, ntk) = kernel(x1, x2; W_std, b_std) of a Myrtle-style network
   whose convolutions share ``W_std``, ``b_std``; differentiable in x1, x2,
-  W_std and b_std through the adjoint kernels."""
+  W_std and b_std through the adjoint kernels.  keep_states: leave the pair
+  states for the backward, where there is room."""
 
   @staticmethod
-  def forward(ctx, x1, x2, W_std, b_std, builder):
+  def forward(ctx, x1, x2, W_std, b_std, builder, keep_states=True):
     kernel_fn = builder(float(W_std), float(b_std))
     x2n = None if x2 is None or x2.numel() == 0 else x2
     keep = []
-    more = ({'_keep': keep} if any(ctx.needs_input_grad[:4]) and
+    more = ({'_keep': keep} if keep_states and
+            any(ctx.needs_input_grad[:4]) and
             isinstance(kernel_fn, stax.AnalyticKernelFn) else {})
     k = kernel_fn(x1.detach(), None if x2n is None else x2n.detach(),
                   ('nngp', 'ntk'), **more)
@@ -490,7 +492,7 @@ class KernelFunction(torch.autograd.Function):
                       device=dev) if need[3] else None
     gx1 = gx1.to(x1.dtype) if need[0] else None
     gx2 = None if ctx.sym or not need[1] else gx2.to(x2.dtype)
-    return gx1, gx2, gW, gb, None
+    return gx1, gx2, gW, gb, None, None
 
 
 def myrtle_builder(depths=(2, 1, 1), readout_W_std=1.0, readout_b_std=0.0):
@@ -508,7 +510,9 @@ def kernel(x1, x2, W_std, b_std, builder):
   """Differentiable (nngp, ntk); pass ``x2=None`` for K(x1, x1)."""
   if x2 is None:
     x2 = torch.empty(0, device=x1.device)
-  return KernelFunction.apply(x1, x2, W_std, b_std, builder)
+  # without gradients nothing is left for a backward
+  return KernelFunction.apply(x1, x2, W_std, b_std, builder,
+                              torch.is_grad_enabled())
 
 
 def krr_loss(x_support, y_support, x_target, y_target, W_std, b_std,
