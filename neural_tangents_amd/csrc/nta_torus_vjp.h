@@ -594,10 +594,13 @@ int vjp_run(const TorusArgs& A, const VjpArgs& V, const float* x1,
   constexpr int Ks = L * H * H;
   constexpr size_t bytes =
       sizeof(float) * vjp_pairs(LW) * (size_t)(body > Ks ? body : Ks);
-  if (bytes > 64 * 1024)
-    (void)hipFuncSetAttribute(
+  if (bytes > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute(
         reinterpret_cast<const void*>(k_torus_vjp<LW, RS, L, NTK, IMG>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess)
+      return set_error((int)e, "nta_torus_vjp: %s", hipGetErrorString(e));
+  }
   const long long blocks =
       (A.np + vjp_pairs(LW) - 1) / vjp_pairs(LW) * V.nsplit;
   hipLaunchKernelGGL((k_torus_vjp<LW, RS, L, NTK, IMG>),
