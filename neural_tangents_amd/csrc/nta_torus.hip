@@ -1,6 +1,7 @@
 // Host side of the register-resident chains (nta_torus.h): geometry, launch
 // shapes, the readout of the partial sums and the C entry points.
 #include <algorithm>
+#include <atomic>
 
 #include "nta_torus.h"
 
@@ -82,25 +83,17 @@ __global__ __launch_bounds__(256) void k_torus_readout(
 // Compute units of the current device (workgroups of a launch are balanced
 // over them).
 int torus_units() {
-  static int cus[16] = {0};
+  static std::atomic<int> cus[16];        // several threads may ask first
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 256;
-  if (cus[dev] == 0) {
-    int v = 0;
+  int v = cus[dev].load(std::memory_order_relaxed);
+  if (v == 0) {
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount,
                               dev) != hipSuccess || v <= 0)
       v = 256;
-    cus[dev] = v;
+    cus[dev].store(v, std::memory_order_relaxed);
   }
-  return cus[dev];
-}
-
-static size_t pool_lds(const TorusGeom& g, int L, bool img) {
-  const size_t x = g.lw == 32 ? 16 * g.PR / 2 * 16 * 2
-                              : (size_t)g.Q * (g.PR / 2) * g.lw * 2;
-  const size_t per = (img ? (size_t)(g.PR + g.TR) * g.lw * 4 : 0) +
-                     (size_t)L * (g.PR + g.TR) * g.lw * 2 + x;
-  return per * (g.lw == 8 ? 4 : 1) * sizeof(float);
+  return v;
 }
 
 // Fills the geometry and the layers' constants; *act receives the kernel's
@@ -245,7 +238,7 @@ static void choose_chunks(TorusArgs& A, const TorusGeom& g) {
     }
     return;
   }
-  const int spw = g.lw == 32 ? 1 : 64 / g.lw;
+  const int spw = 64 / g.lw;
   A.ns = A.P * ((A.Q + spw - 1) / spw);
   const long long room = 16LL * torus_units();   // waves in flight
   long long best = -1;
@@ -253,11 +246,8 @@ static void choose_chunks(TorusArgs& A, const TorusGeom& g) {
     if (cs > A.ns) cs = A.ns;
     const int nc = (A.ns + cs - 1) / cs;
     const long long jobs = A.np * nc;
-    // rounds of waves x slices of a wave, in quarters of a slice's time, the
-    // last round counted by its share
-    const long long full = jobs / room, rest = jobs % room;
-    const long long cost =
-        (4 * cs + 1) * (full + (rest > room / 2 ? 1 : (rest ? 1 : 0)));
+    // rounds of waves x slices of a wave, in quarters of a slice's time
+    const long long cost = (4 * cs + 1) * ((jobs + room - 1) / room);
     if (best < 0 || cost < best) {
       best = cost;
       A.cs = cs;
@@ -279,7 +269,8 @@ extern "C" int nta_torus_supported(int H, int W, int C, int L, int pool,
     return 0;
   if (L < 1 || L > kTorusMaxL || C < 0 || C > 4) return 0;
   if (C == 0 && g.lw == 32) return 0;
-  if (pool && (H < 2 || W < 2 || pool_lds(g, L, C > 0) > 160 * 1024))
+  if (pool && (H < 2 || W < 2 || torus_pool_lds(g.lw, g.Q, g.PR, g.TR, L, C > 0) >
+                                160 * 1024))
     return 0;
   return 1;
 }
@@ -367,7 +358,7 @@ extern "C" int nta_torus_pool(const float* x1, const float* x2, int n1,
   A.Qn = go.Q;
   A.out_scale *= 1.0 / 16.0;
   const int Ph = A.P / 2;
-  const size_t lds = pool_lds(g, L, img);
+  const size_t lds = torus_pool_lds(g.lw, g.Q, g.PR, g.TR, L, img);
   const long long per_cu =
       g.lw == 32 ? 1 : std::max<long long>(1, std::min<long long>(
                            4, (160 * 1024) / (long long)lds));
