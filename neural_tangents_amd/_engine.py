@@ -348,8 +348,7 @@ def _kept_states(segs, pairs, want_ntk, dev):
   """Empty (nngp, ntk) states of all pairs before every segment but the first,
   counted against KEEP_BYTES while anything holds them, or None if there is no
   room."""
-  sizes = [_lib.value('nta_torus_state_floats', s.H, s.W) for s in segs[1:]]
-  need = 4 * pairs * sum(sizes) * (2 if want_ntk else 1)
+  need = 4 * pairs * sum(s.state for s in segs[1:]) * (2 if want_ntk else 1)
   with _kept_lock:
     entry = _kept.setdefault(dev, [0, []])
     if entry[0] + need > KEEP_BYTES:
@@ -912,6 +911,8 @@ class Segment:
   flags: int
   pool: bool                       # AvgPool 2x2 into the next segment
   crop: Tuple[int, int]            # last segment: elements the mean keeps
+  state: int                       # floats of a pair's state before it
+  table: int                       # floats of an image's and layer's table
 
   def layer_bytes(self, first: bool) -> int:
     """HBM bytes per pair and tensor of a schedule that runs every layer as
@@ -972,7 +973,9 @@ def _torus_segments(plan: Plan, in_shape) -> Optional[List[Segment]]:
                       len(layers), int(not last), flags):
       return None
     segs.append(Segment(H, W, len(layers), wb, flags, not last,
-                        tuple(keep) if last else (H, W)))
+                        tuple(keep) if last else (H, W),
+                        _lib.value('nta_torus_state_floats', H, W),
+                        _lib.value('nta_torus_table_floats', H, W, 0)))
     layers = []
     H, W = H // 2, W // 2
   return segs or None
@@ -990,15 +993,13 @@ def _torus_bands(segs) -> List[int]:
 
 def _torus_state(n, seg, dev):
   """An empty state of n pairs before seg."""
-  return torch.empty((n, _lib.value('nta_torus_state_floats', seg.H, seg.W)),
-                     dtype=torch.float32, device=dev)
+  return torch.empty((n, seg.state), dtype=torch.float32, device=dev)
 
 
 def _torus_tables(segs, n, dev):
   """Empty normaliser tables of n images, per segment."""
-  return [torch.empty((s.L, n, _lib.value('nta_torus_table_floats', s.H, s.W,
-                                          0)),
-                      dtype=torch.float32, device=dev) for s in segs]
+  return [torch.empty((s.L, n, s.table), dtype=torch.float32, device=dev)
+          for s in segs]
 
 
 def _torus_images(x1, x2, most):
@@ -1079,19 +1080,16 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
   def state(n, seg):
     return _torus_state(n, seg, dev)
 
-  # a segment's input and output state
-  floats = [0] + [_lib.value('nta_torus_state_floats', s.H, s.W)
-                  for s in segs[1:]] + [0]
-  most = max(1, tile_bytes // max(1, 4 * max(map(sum, zip(floats,
-                                                          floats[1:])))))
+  # the pooled states, of which a segment holds its input and output
+  big = max((s.state for s in segs[1:]), default=0)
   coef = plan.head_coef if want_cov else None
-  parts = _torus_images(x1, x2, most)
-  if len(parts) == 1:
+  most = max(1, tile_bytes // max(1, 8 * big))
+  if nimg <= most:
     tabs, _, _, cov = _torus_selfs(segs, x1, x2, stream, coef)
   else:
     tabs = _torus_tables(segs, nimg, dev)
     cov = empty(nimg) if want_cov else None
-    for xa, xb, at, n in parts:
+    for xa, xb, at, n in _torus_images(x1, x2, most):
       part, _, _, pcov = _torus_selfs(segs, xa, xb, stream, coef)
       for t, p in zip(tabs, part):
         t[:, at:at + n] = p
@@ -1104,8 +1102,7 @@ def _run_torus(plan: Plan, segs, x1, x2, want_ntk, want_cov, tile_bytes,
   mode = (_lib.TORUS_UPPER if x2 is None else 0) | (
       _lib.NTK if want_ntk else 0)
   nt = 2 if want_ntk else 1
-  per = max([4 * nt * 2 * _lib.value('nta_torus_state_floats', s.H, s.W)
-             for s in segs[1:]], default=0)
+  per = 4 * nt * 2 * big
   tile = min(pairs, max(1, tile_bytes // per) if per else 1 << 20)
   held = None
   if keep is not None and tile == pairs:

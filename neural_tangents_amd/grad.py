@@ -326,9 +326,8 @@ def _torus_vjp(plan, segs, x1, x2, g_nngp, g_ntk, tile_pairs, kept):
   band = [b if s.pool else -1
           for b, s in zip(_engine._torus_bands(segs), segs)]
   first = [sum(s.L for s in segs[:k]) for k in range(K)]
-  per = sum(work_bytes(k, 1, band[k]) + 8 * _lib.value(
-      'nta_torus_state_floats', s.H, s.W) * (k > 0)
-      for k, s in enumerate(segs))
+  per = sum(work_bytes(k, 1, band[k]) + 8 * s.state * (k > 0)
+            for k, s in enumerate(segs))
   parts = _engine._torus_images(x1, x2, max(1, SELF_BYTES // per))
   if len(parts) == 1:
     ftabs, tabs, selfs, _ = _engine._torus_selfs(segs, x1, x2, stream,
