@@ -65,23 +65,27 @@ def test_self_covariance(side):
 
 @pytest.mark.parametrize('side', [8, 16, 32])
 @pytest.mark.parametrize('same', [True, False])
-def test_gradients(side, same):
-  """Input gradients of images times s are s times those of the images."""
+@pytest.mark.parametrize('b', [0.0, 0.1])
+def test_gradients(side, same, b):
+  """Images and b_std times s: K times s^2, its gradients in them times s, in
+  W_std times s^2."""
   xs = _images(side)
   s = 2.0 ** -30
 
   def run(scale):
-    a, b = (x.mul(scale).requires_grad_() for x in xs)
+    xa, xb = (x.mul(scale).requires_grad_() for x in xs)
     W = torch.tensor(2.0 ** 0.5, device='cuda', requires_grad=True)
-    n, t = grad.kernel(a, None if same else b, W, 0.0,
+    bs = torch.tensor(b * scale, device='cuda', requires_grad=True)
+    n, t = grad.kernel(xa, None if same else xb, W, bs,
                        grad.myrtle_builder((2, 1, 1)))
-    return torch.autograd.grad((n + t).sum(), (a, W) if same else (a, b, W))
+    return torch.autograd.grad((n + t).sum(),
+                               [W, bs, xa] + ([] if same else [xb]))
   want, got = run(1.0), run(s)
-  for g, w in zip(got[:-1], want[:-1]):
+  for g, w in zip(got[2:], want[2:]):
     assert torch.equal(g.double() / s, w.double())
-  # W_std's comes from FP64 sums of FP32 products
-  assert abs(float(got[-1]) / s ** 2 - float(want[-1])) <= 1e-6 * abs(
-      float(want[-1]))
+  # FP64 sums of FP32 products
+  for g, w, fac in ((got[0], want[0], s * s), (got[1], want[1], s)):
+    assert abs(float(g) / fac - float(w)) <= 1e-6 * abs(float(w))
 
 
 @pytest.mark.parametrize('n1,n2', [(5, 9), (90, 0), (1500, 1400)])
