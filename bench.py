@@ -326,7 +326,6 @@ def m10_result(steps):
           'path_pct_hbm_peak': 100.0 * bpp * value / 1e9 / HBM_PEAK_GBS,
           'dominant_kernel': dom,
           'dominant_gbs_canonical': table[dom]['gbs'],
-          'dominant_frac_hbm_peak': table[dom]['gbs'] / HBM_PEAK_GBS,
           'note': SCHEDULE_NOTES.get(dom, ''),
           'kernels': table}
 
@@ -377,8 +376,8 @@ SCHEDULE_NOTES = {
         'achieved counts the per-layer schedule\'s bytes for those layers '
         '(the 32^4 states written and read back, the pooled state written); '
         'the kernel forms none of them, so measured HBM traffic is far below; '
-        'its bound is the vector ALU (valu_busy_frac, from rocprofv3 '
-        'counters)',
+        'its bound is the vector ALU (share of issue slots, from committed '
+        'rocprofv3 counters)',
     'nta_first3_pool_stage':
         'first three stages fused ([Conv-Relu] x 3 - AvgPool, Myrtle-10): '
         'achieved counts the per-layer schedule\'s bytes for those three '
@@ -389,8 +388,7 @@ SCHEDULE_NOTES = {
         'counts the per-layer schedule\'s bytes for those two kernels (the '
         'first stage state written and read back, the pooled state written); '
         'the kernel never materialises the first stage, so traffic (measured '
-        'HBM bytes) is far below them; its bound is the vector ALU '
-        '(valu_busy_frac, from rocprofv3 counters)',
+        'HBM bytes) is far below them; its bound is the vector ALU',
 }
 
 
@@ -451,12 +449,31 @@ def readme_cnn21_result(n_flat=512, n_gap=16, steps=3):
   return res
 
 
-def valu_busy(kernel):
+def valu_issue(kernel):
+  """Share of the vector issue slots that ``kernel`` uses (SQ_INSTS_VALU x 4
+  cycles per SIMD and GPU-active cycle), from the committed counters, or
+  None."""
   d = _load_json(VALU_FILE)
   try:
-    return d['kernels'][kernel]['valu_busy_frac']
+    return d['kernels'][kernel]['valu_issue_frac']
   except (TypeError, KeyError):
     return None
+
+
+def roofline(name, achieved_gbs, avg_ms, avg_bytes, traffic):
+  """The dominant kernel against what bounds it: the vector ALU for launches
+  that fuse several layers (their per-layer bytes, which most of them never
+  move, stand beside it), HBM otherwise."""
+  out = {'kernel': name, 'avg_launch_ms': avg_ms, 'traffic': traffic,
+         'alg_bytes_per_launch': avg_bytes,
+         'note': SCHEDULE_NOTES.get(name, '')}
+  if name.startswith(('nta_first', 'nta_torus')):
+    frac = valu_issue(name)
+    return {'bound': 'valu', 'achieved': frac, 'peak': 1.0,
+            'unit': 'share of vector issue slots', 'frac': frac,
+            'canonical_gbs': achieved_gbs, **out}
+  return {'bound': 'hbm', 'achieved': achieved_gbs, 'peak': HBM_PEAK_GBS,
+          'unit': 'GB/s', 'frac': achieved_gbs / HBM_PEAK_GBS, **out}
 
 
 def main():
@@ -539,8 +556,6 @@ def main():
   value = pairs * args.steps / elapsed
   bpp = canonical_bytes_per_pair(depths, side)
   log(f'{args.workload}: {value:.0f} pairs/s')
-  fused = dom_name.startswith(('nta_first_pool_stage', 'nta_torus'))
-  vb = valu_busy(dom_name) if fused else None
 
   out = {
       'metric': 'Myrtle NTK pairs/sec + %HBM peak',
@@ -560,14 +575,9 @@ def main():
                  'get': ['nngp', 'ntk'], 'parallelism': 'single GPU'},
       'path_gbs_canonical': bpp * value / 1e9,
       'path_pct_hbm_peak': 100.0 * bpp * value / 1e9 / HBM_PEAK_GBS,
-      'roofline': {'bound': 'hbm', 'limiter': 'valu' if fused else 'hbm',
-                   'kernel': dom_name,
-                   'achieved': achieved, 'peak': HBM_PEAK_GBS,
-                   'unit': 'GB/s', 'frac': achieved / HBM_PEAK_GBS,
-                   'traffic': traffic, 'avg_launch_ms': avg_ms,
-                   'alg_bytes_per_launch': avg_bytes,
-                   'valu_busy_frac': vb,
-                   'note': SCHEDULE_NOTES.get(dom_name, '')},
+      'path_note': 'bytes of the per-layer schedule; most are never moved, so '
+                   'the share can pass 100%',
+      'roofline': roofline(dom_name, achieved, avg_ms, avg_bytes, traffic),
       'kernels': kernel_table(per, args.steps),
   }
   got = (k.nngp.cpu().numpy(), k.ntk.cpu().numpy())
