@@ -92,14 +92,14 @@ __host__ __device__ constexpr int vjp_parked(int L, bool ntk, bool img) {
 // over the waves in LDS, in a fixed order, at the end.
 // Bound: the vector ALU (about 140 instructions per element of a two-layer
 // segment from images, two waves a SIMD).  512 pairs of 32x32 images, 2
-// layers: 2.76 ms here and 0.35 ms in k_torus_pixels (3.35 ms while the layer
+// layers: 2.8 ms here and 0.35 ms in k_torus_pixels (3.35 ms while the layer
 // before the last was mapped again on the way back instead of keeping s and
 // pk, cuts were worked out per stencil and s and 1 / s took a root and a
 // reciprocal); with the pixels' sums in the same registers 5.7 ms (336 bytes a
 // lane spilled).  The per-layer kernels of the general path stream states of
 // 4 MiB a pair and tensor through k_relu_bwd_rows, the stencils and two GEMMs:
 // the gradients of 20 x 20 and 20 x 64 pairs through Myrtle-5 took 43.2 ms
-// with them, 15.9 ms with these (forward included).
+// with them, 16.0 ms with these (forward included).
 // part[pair][split]: side i, then side j: [L][H W]; wbp[pair][split][L][2].
 // gin: the cotangent of the input, from a state in its layout, from images
 // (of the input covariance) [pair][e - e0][d - d0][h][w].
